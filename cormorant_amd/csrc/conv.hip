@@ -17,9 +17,10 @@
 //     GEMM Y[n] = W[out_ch][in_ch] x X[n][in_ch][h*w] on the int8-limb MFMA core;
 //   * any other: implicit GEMM on the same core, im2col gathered straight from
 //     NCHW x while the B tile is built (no im2col buffer);
-//   * depthwise (is_depthwise = 1, weights [out_ch][1][kh][kw]): LDS band kernel
-//     (rows too wide for it: one thread per output), uint32 wrapping accumulator
-//     (ConvKernel.cpp:251-319).
+//   * depthwise (is_depthwise = 1, weights [out_ch][1][kh][kw]): 3x3 and 5x5
+//     windows streamed through registers (conv_dw.hip), others on the LDS band
+//     kernel (rows too wide for it: one thread per output), uint32 wrapping
+//     accumulator (ConvKernel.cpp:251-319).
 // All paths: acc = wrap32((has_bias ? bias << 8 : 0) + sum x*w), y = sat16(acc >> 8),
 // then the optional fused epilogue (Add of a same-shaped tensor, Relu / Relu6).
 #include "cm_internal.h"
@@ -51,6 +52,10 @@ int cm_conv_pgemm_launch(const int16_t* x, const int16_t* w, const int16_t* bias
                          uint32_t out_ch, uint32_t out_h, uint32_t out_w, uint32_t kh, uint32_t kw,
                          uint32_t sh, uint32_t sw, uint32_t dh, uint32_t dw, uint32_t pad_top,
                          uint32_t pad_left, const cm_epilogue_t* epi, const LaunchCtx& lc);
+int cm_conv_dw_rows_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y, uint32_t batch,
+                           uint32_t in_ch, uint32_t in_h, uint32_t in_w, uint32_t out_ch, uint32_t out_h,
+                           uint32_t out_w, uint32_t kh, uint32_t kw, uint32_t sh, uint32_t sw, uint32_t dh,
+                           uint32_t dw, uint32_t pt, uint32_t pl, const EpiArgs& epi, hipStream_t s);
 
 namespace {
 
@@ -585,6 +590,9 @@ int cm_conv_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int1
     if (is_dw) {
         const uint64_t total = (uint64_t)batch * out_ch * out_h * out_w;
         if (total == 0 || lc.need) return CM_OK;
+        const int rc = cm_conv_dw_rows_launch(x, w, b, y, batch, in_ch, in_h, in_w, out_ch, out_h, out_w, kh, kw,
+                                              sh, sw, dh, dw, pad_top, pad_left, ea, s);
+        if (rc != 1) return rc;
         DwBand bg{};
         bg.x = x; bg.w = w; bg.bias = b; bg.y = y; bg.epi = ea;
         bg.C = in_ch; bg.M = out_ch; bg.H = in_h; bg.W = in_w; bg.OH = out_h; bg.OW = out_w;
