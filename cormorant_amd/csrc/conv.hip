@@ -2,6 +2,9 @@
 //
 // Dispatch (standard convolutions, first match):
 //   * few output channels, K <= 32, many pixels: direct vector-ALU kernel;
+//   * 1x1 / stride 1 / no padding, 8 to 512 channels (above 256: larger layers
+//     only): limb planes of a few pixel groups in LDS, 16-byte accesses of eight
+//     pixels throughout (conv_pws.hip);
 //   * strided windows of 2..32 taps, small layers (<= 2^19 outputs, K <= 2048): one
 //     block of four waves per 32x32 output tile, the reduction split over the
 //     waves, fragments loaded straight into registers (conv_rk.hip);
@@ -10,10 +13,10 @@
 //     LDS, weights pre-split into limb planes; conv_pgemm.hip);
 //   * 3x3, <= 64 channels in and out, stride 1 or 2: conv_patch (input patch and
 //     all weights in LDS);
-//   * 1x1 / stride 1 / no padding, small layers (<= 2^21 outputs, in_ch <= 512):
+//   * other 1x1 / stride 1 / no padding, small layers (<= 2^21 outputs, in_ch <= 512):
 //     one wave per 32x32 output tile, fragments loaded straight into registers,
 //     no LDS (conv_pw.hip);
-//   * 1x1 / stride 1 / no padding, planes that fill 128-column tiles: batched
+//   * other 1x1 / stride 1 / no padding, planes that fill 128-column tiles: batched
 //     GEMM Y[n] = W[out_ch][in_ch] x X[n][in_ch][h*w] on the int8-limb MFMA core;
 //   * any other: implicit GEMM on the same core, im2col gathered straight from
 //     NCHW x while the B tile is built (no im2col buffer);
@@ -39,6 +42,8 @@ int cm_conv_pointwise_launch(const int16_t* x, const int16_t* w, const int16_t* 
 int cm_conv_pw_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y,
                       uint32_t batch, uint32_t in_ch, uint32_t out_ch, uint32_t hw,
                       const cm_epilogue_t* epi, const LaunchCtx& lc);
+int cm_conv_pws_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y, uint32_t batch,
+                       uint32_t in_ch, uint32_t out_ch, uint32_t hw, const cm_epilogue_t* epi, const LaunchCtx& lc);
 bool cm_conv_rk_takes(uint32_t batch, uint32_t in_ch, uint32_t in_h, uint32_t in_w, uint32_t out_ch,
                       uint32_t out_h, uint32_t out_w, uint32_t kh, uint32_t kw, uint32_t sh, uint32_t sw,
                       uint32_t dh, uint32_t dw, uint32_t pad_top, uint32_t pad_left);
@@ -646,6 +651,20 @@ int cm_conv_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int1
             default: return launch_direct<32>(g, s);
         }
     }
+    // 1x1 / stride 1 / no padding (conv_pws.hip).  Up to 256 channels its blocks are
+    // small enough for any layer: 64 -> 64 at 16 x 28 x 28 4.5 us against conv_pw's
+    // 5.3, 128 -> 256 at 28 x 28 4.8 against conv_rk's 5.3 (small planes that are not
+    // whole eight-pixel groups tie: 160 -> 320 at 16 x 7 x 7 5.6 against 5.5).  Above,
+    // a block needs the CU's LDS, so layers have to fill the GPU: 512 -> 512 at
+    // 16 x 14 x 14 14.3 against 20.5, but 15.4 against 10.4 at 7 x 7.
+    const uint64_t hw = (uint64_t)in_h * in_w;
+    const bool pointwise = kh == 1 && kw == 1 && sh == 1 && sw == 1 && pad_top == 0 && pad_left == 0 &&
+                           out_h == in_h && out_w == in_w && hw <= 0x7FFFFFFFull;
+    const uint64_t outs = npix * out_ch;
+    if (pointwise && (in_ch <= 256 ? hw % 8 == 0 || outs > (1u << 19) : outs > (1u << 20))) {
+        const int rc = cm_conv_pws_launch(x, w, b, y, batch, in_ch, out_ch, (uint32_t)hw, epi, lc);
+        if (rc != 1) return rc;
+    }
     // Small layers: the register-only kernel with the reduction split over a
     // block's waves (conv_rk.hip)
     if (cm_conv_rk_takes(batch, in_ch, in_h, in_w, out_ch, out_h, out_w, kh, kw, sh, sw, dh, dw, pad_top,
@@ -676,14 +695,11 @@ int cm_conv_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int1
         const int rc = try_patch();
         if (rc != 1) return rc;
     }
-    // 1x1 / stride 1 / no padding: small layers on the register-only MFMA kernel
-    // (conv_pw.hip); else one GEMM per image, when an image's pixels fill its
+    // Other 1x1 / stride 1 / no padding layers: small ones on the register-only MFMA
+    // kernel (conv_pw.hip); else one GEMM per image, when an image's pixels fill its
     // 128-column tiles to at least 80 %; small planes (e.g. 7x7, 14x14) go
     // through the gather path, whose columns run across images
-    const uint64_t hw = (uint64_t)in_h * in_w;
     const uint64_t tiles = (hw + 127) / 128;
-    const bool pointwise = kh == 1 && kw == 1 && sh == 1 && sw == 1 && pad_top == 0 && pad_left == 0 &&
-                           out_h == in_h && out_w == in_w && hw <= 0x7FFFFFFFull;
     if (pointwise) {
         const int rc = cm_conv_pw_launch(x, w, b, y, batch, in_ch, out_ch, (uint32_t)hw, epi, lc);
         if (rc != 1) return rc;

@@ -42,11 +42,11 @@ typedef short v2s __attribute__((ext_vector_type(2)));
 typedef unsigned int v2u __attribute__((ext_vector_type(2)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
 
-// From this size on x and y together no longer stay in the Infinity Cache (256 MB
-// on an MI355X) until they are used next, so y is stored past it: 31.2 -> 26.9 us
-// at 154 MB, but 12.4 -> 14.4 at 58 MB and 13.8 -> 27.4 at 38 MB (rows of 56 bytes:
+// From this size on (a third of the MI355X's 256 MB Infinity Cache) x and y
+// together no longer stay there until they are used next, and y is stored past
+// it: 31.2 -> 26.9 us at 154 MB, 17.1 -> 16.1 at 96 MB, but 12.4 -> 14.4 at 58 MB and 13.8 -> 27.4 at 38 MB (rows of 56 bytes:
 // partial lines), which the cache holds.  Whole 16-byte rows only.
-constexpr uint64_t kStreamBytes = 128ull << 20;
+constexpr uint64_t kStreamBytes = 80ull << 20;
 
 struct DwRows {
     const int16_t* x;
