@@ -26,10 +26,19 @@
 // layouts and their bank conflicts).  The next tile's loads are issued before the MFMA phase; loads are
 // unconditional (out-of-range elements are zeroed by the buffer range check
 // or by a select), so all of a tile's loads are in flight at once.
+//
+// Dense products run on gemm_rg.hip when they fit it; here stay those with K above
+// 32768 (the fold), fewer than 8 k or 4 columns, more than 2^30 elements, and the
+// pointwise convolutions that reach launch_gemm (a bias per row).
 #include <type_traits>
 
 #include "cm_internal.h"
 #include "q88.h"
+
+uint32_t cm_gemm_rg_splits(uint32_t n, uint32_t m, uint32_t nk, uint32_t splits);
+int cm_gemm_rg_launch(const int16_t* a, const int16_t* b, int16_t* c, uint32_t n, uint32_t k, uint32_t m,
+                      uint64_t a_bs, uint64_t b_bs, uint64_t c_bs, uint32_t z, uint32_t* ws, uint32_t steps,
+                      uint32_t ws_ld, const EpiArgs& epi, hipStream_t s);
 
 namespace {
 
@@ -951,6 +960,19 @@ uint32_t choose_splits(uint32_t tiles, uint32_t nk_all) {
     return sp < 2 ? 1 : sp;
 }
 
+// The second pass of a split launch: sums the partials, adds bias and epilogue.
+int launch_splits(const GemmArgs& g, uint32_t splits, hipStream_t s, bool conv) {
+    ReduceArgs r{};
+    r.ws = g.ws; r.rows = g.rows; r.cols = g.cols; r.ws_ld = g.ws_ld;
+    r.div_q = make_fastdiv(g.ws_ld / 4u);
+    r.bias = g.bias; r.y = g.c;
+    r.conv = conv; r.P = g.P; r.div_p = g.div_p;
+    r.y_img = g.y_img; r.ldc = g.ldc; r.epi = g.epi;
+    const uint64_t chunks = (uint64_t)g.rows * (g.ws_ld / 4u);
+    const dim3 rgrid((uint32_t)cm_grid_blocks(chunks, kReduceThreads, 4096));
+    return launch_reduce<2>(splits, rgrid, s, r);
+}
+
 inline bool aligned(const void* p, uintptr_t n) { return ((uintptr_t)p & (n - 1)) == 0; }
 
 template <int MODE>
@@ -999,6 +1021,21 @@ int launch_gemm(GemmArgs& g0, uint32_t zdim, const LaunchCtx& lc, const char* na
     } else if (lc.need) {
         return CM_OK;
     }
+    if constexpr (MODE == B_DENSE) {
+        if (!g.bias && !fold) {
+            uint32_t sp = 1, steps = 0;
+            if (splits > 1) {
+                const uint32_t nk_all = (g.k + BK - 1) / BK;
+                steps = (nk_all + cm_gemm_rg_splits(g.rows, g.cols, nk_all, splits) - 1) /
+                        cm_gemm_rg_splits(g.rows, g.cols, nk_all, splits);
+                sp = (nk_all + steps - 1) / steps;   // no empty split
+            }
+            const int rc = cm_gemm_rg_launch(g.a, g.b, g.c, g.rows, g.k, g.cols, g.a_bs, g.b_bs, g.c_bs,
+                                             splits > 1 ? sp : grid.z, sp > 1 ? g.ws : nullptr, steps, g.ws_ld, g.epi, s);
+            if (rc < 0) return rc;
+            if (rc == 0) return sp > 1 ? launch_splits(g, sp, s, false) : rc;
+        }
+    }
     const bool bias = g.bias != nullptr && splits == 1;
     // widest output / Add access that keeps alignment and stays in one image row run
     g.out_w = 8;
@@ -1038,18 +1075,8 @@ int launch_gemm(GemmArgs& g0, uint32_t zdim, const LaunchCtx& lc, const char* na
     }
 #undef CM_GEMM_BIAS
 #undef CM_GEMM_LAUNCH
-    if (splits == 1) return cm_check_launch(name);
     const int rc = cm_check_launch(name);
-    if (rc) return rc;
-    ReduceArgs r{};
-    r.ws = g.ws; r.rows = g.rows; r.cols = g.cols; r.ws_ld = g.ws_ld;
-    r.div_q = make_fastdiv(g.ws_ld / 4u);
-    r.bias = g.bias; r.y = g.c;
-    r.conv = MODE != B_DENSE; r.P = g.P; r.div_p = g.div_p;
-    r.y_img = g.y_img; r.ldc = g.ldc; r.epi = g.epi;
-    const uint64_t chunks = (uint64_t)g.rows * (g.ws_ld / 4u);
-    const dim3 rgrid((uint32_t)cm_grid_blocks(chunks, kReduceThreads, 4096));
-    return launch_reduce<2>(splits, rgrid, s, r);
+    return rc || splits == 1 ? rc : launch_splits(g, splits, s, MODE != B_DENSE);
 }
 
 }  // namespace
