@@ -197,6 +197,17 @@ __global__ __launch_bounds__(kThreads) void conv_dw_rows(DwRows g) {
     const v2s lo = {(short)q88::act_lo(g.epi.act), (short)q88::act_lo(g.epi.act)};
     const v2s hi = {(short)q88::act_hi(g.epi.act), (short)q88::act_hi(g.epi.act)};
 
+    // the Add's operands of every row, ahead of the first store: a load between two
+    // stores would wait for the store before it
+    uint32_t add[U][OPL / 2];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int q = 0; q < OPL / 2; ++q) add[u][q] = 0u;
+    if (g.epi.add_mode == 1u) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) load_run<OPL>(ar, r0 + u < g.OH ? yoff + u * yrow : kOob, on, add[u]);
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const uint32_t off = r0 + u < g.OH ? yoff + u * yrow : kOob;
@@ -217,17 +228,9 @@ __global__ __launch_bounds__(kThreads) void conv_dw_rows(DwRows g) {
 #pragma unroll
         for (int q = 0; q < OPL / 2; ++q)
             out[q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pk_i16(acc[2 * q] >> 8, acc[2 * q + 1] >> 8));
-        if (g.epi.add_mode == 1u) {
-            uint32_t add[OPL / 2];
-            load_run<OPL>(ar, off, on, add);
-#pragma unroll
-            for (int q = 0; q < OPL / 2; ++q)
-                out[q] = __builtin_bit_cast(uint32_t, __builtin_elementwise_add_sat(
-                    __builtin_bit_cast(v2s, out[q]), __builtin_bit_cast(v2s, add[q])));
-        }
 #pragma unroll
         for (int q = 0; q < OPL / 2; ++q) {
-            const v2s v = __builtin_bit_cast(v2s, out[q]);
+            const v2s v = __builtin_elementwise_add_sat(__builtin_bit_cast(v2s, out[q]), __builtin_bit_cast(v2s, add[u][q]));
             out[q] = __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_elementwise_max(v, lo), hi));
         }
         store_run<OPL, NT ? kNonTemporal : 0>(yr, off, on, out);

@@ -34,6 +34,7 @@
 #include "cm_internal.h"
 #include "limbs.h"
 #include "q88.h"
+#include "runs.h"
 
 #include <algorithm>
 
@@ -60,41 +61,11 @@ struct RgArgs {
 using limbs::bsum;
 using limbs::hi4;
 using limbs::lo4;
+using runs::load_head;
+using runs::store_head;
 
 __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
     return __builtin_amdgcn_perm(hi, lo, sel);
-}
-
-// The first n of eight int16 values at byte offset `off`.
-__device__ __forceinline__ v4u load_head(__amdgpu_buffer_rsrc_t rs, uint32_t off, uint32_t n) {
-    if (n == 8u) return __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
-    v4u d;
-#pragma unroll
-    for (uint32_t q = 0; q < 4; ++q) {
-        const uint32_t lo = __builtin_amdgcn_raw_buffer_load_b16(rs, 2u * q < n ? off + 4u * q : kOob, 0, 0);
-        const uint32_t hi = __builtin_amdgcn_raw_buffer_load_b16(rs, 2u * q + 1u < n ? off + 4u * q + 2u : kOob, 0, 0);
-        d[q] = (lo & 0xFFFFu) | hi << 16;
-    }
-    return d;
-}
-__device__ __forceinline__ void store_head(__amdgpu_buffer_rsrc_t rs, uint32_t off, uint32_t n, v4u d) {
-    if (n == 8u) {
-        __builtin_amdgcn_raw_buffer_store_b128(d, rs, off, 0, 0);
-        return;
-    }
-    uint32_t a = d[0], b = d[1];
-    if (n & 4u) {
-        __builtin_amdgcn_raw_buffer_store_b64(v2u{a, b}, rs, off, 0, 0);
-        a = d[2];
-        b = d[3];
-        off += 8u;
-    }
-    if (n & 2u) {
-        __builtin_amdgcn_raw_buffer_store_b32(a, rs, off, 0, 0);
-        a = b;
-        off += 4u;
-    }
-    if (n & 1u) __builtin_amdgcn_raw_buffer_store_b16((uint16_t)a, rs, off, 0, 0);
 }
 
 // WR x WC waves of 32 x 64 outputs; KS groups of them take every KS-th k step and
@@ -425,6 +396,23 @@ __global__ __launch_bounds__(WR * WC * KS * 64, 2) void gemm_rg(RgArgs g) {
                 v[e][t] = ((((uint32_t)hh[q][i][ee] << 8) + (uint32_t)mid[q][i][ee]) << 8) + (uint32_t)ll[q][i][ee];
             }
     };
+    // The Add's operands of every output, ahead of the first store: a load between two
+    // stores would wait for the store before it
+    v4u addv[2][2];
+#pragma unroll
+    for (uint32_t i = 0; i < 2; ++i)
+#pragma unroll
+        for (uint32_t e = 0; e < 2; ++e) addv[i][e] = v4u{0u, 0u, 0u, 0u};
+    if (g.epi.add_mode && !g.ws) {
+#pragma unroll
+        for (uint32_t i = 0; i < 2; ++i)
+#pragma unroll
+            for (uint32_t e = 0; e < 2; ++e) {
+                const uint32_t r = row0 + wr * 32u + i * 16u + er16, col = col0 + wc * 64u + (4u * e + ekg) * 8u;
+                const uint32_t cnt = r < g.n && col < g.m ? min(8u, g.m - col) : 0u;
+                addv[i][e] = load_head(er, ((g.epi.add_mode == 1u ? r * g.m : 0u) + col) * 2u, cnt);
+            }
+    }
     // k groups: group kz finishes row tile kz, the other one hands it its sums
     uint32_t* ex = reinterpret_cast<uint32_t*>(lds_all);
     if constexpr (KS == 2) {
@@ -469,8 +457,7 @@ __global__ __launch_bounds__(WR * WC * KS * 64, 2) void gemm_rg(RgArgs g) {
                 continue;
             }
             const uint32_t cnt = min(8u, g.m - col), off = (r * g.m + col) * 2u;
-            v4u add = v4u{0u, 0u, 0u, 0u};
-            if (g.epi.add_mode) add = load_head(er, g.epi.add_mode == 1u ? off : col * 2u, cnt);
+            const v4u add = addv[i][e];
             v4u out;
 #pragma unroll
             for (uint32_t q = 0; q < 4; ++q) {
