@@ -2,6 +2,8 @@
 //
 // Dispatch (standard convolutions, first match):
 //   * few output channels, K <= 32, many pixels: direct vector-ALU kernel;
+//   * at most four input channels, windows of >= 2 taps, dilation 1, stride 1 or 2:
+//     k chunks of four neighbouring columns times four channels (conv_sc.hip);
 //   * 1x1 / stride 1 / no padding, 8 to 512 channels (above 256: larger layers
 //     only): limb planes of a few pixel groups in LDS, 16-byte accesses of eight
 //     pixels throughout (conv_pws.hip);
@@ -42,6 +44,11 @@ int cm_conv_pointwise_launch(const int16_t* x, const int16_t* w, const int16_t* 
 int cm_conv_pw_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y,
                       uint32_t batch, uint32_t in_ch, uint32_t out_ch, uint32_t hw,
                       const cm_epilogue_t* epi, const LaunchCtx& lc);
+int cm_conv_sc_launch(const int16_t* x, const int16_t* w, const uint8_t* wpk, uint32_t wpk_bytes, uint32_t tb,
+                      uint32_t steps, const int16_t* bias, int16_t* y, uint32_t batch, uint32_t in_ch, uint32_t in_h,
+                      uint32_t in_w, uint32_t out_ch, uint32_t out_h, uint32_t out_w, uint32_t kh, uint32_t kw,
+                      uint32_t sh, uint32_t sw, uint32_t dh, uint32_t dw, uint32_t pt, uint32_t pl,
+                      const EpiArgs& epi, hipStream_t s);
 int cm_conv_pws_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* y, uint32_t batch,
                        uint32_t in_ch, uint32_t out_ch, uint32_t hw, const cm_epilogue_t* epi, const LaunchCtx& lc);
 bool cm_conv_rk_takes(uint32_t batch, uint32_t in_ch, uint32_t in_h, uint32_t in_w, uint32_t out_ch,
@@ -650,6 +657,14 @@ int cm_conv_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int1
             case 24: return launch_direct<24>(g, s);
             default: return launch_direct<32>(g, s);
         }
+    }
+    // At most four input channels (conv_sc.hip), where the direct kernel does not take
+    // the layer (3 -> 32, 3x3 stride 2 at 16 x 299 x 299: 19.5 us there, 23.3 here).  The
+    // reported workspace stays the patch GEMM's, which packs for other shapes too.
+    if (in_ch <= 4 && !lc.need) {
+        const int rc = cm_conv_sc_launch(x, w, nullptr, 0, 0, 0, b, y, batch, in_ch, in_h, in_w, out_ch, out_h, out_w,
+                                         kh, kw, sh, sw, dh, dw, pad_top, pad_left, ea, s);
+        if (rc != 1) return rc;
     }
     // 1x1 / stride 1 / no padding (conv_pws.hip).  Up to 256 channels its blocks are
     // small enough for any layer: 64 -> 64 at 16 x 28 x 28 4.5 us against conv_pw's

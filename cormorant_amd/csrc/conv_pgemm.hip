@@ -44,6 +44,12 @@
 #include "cm_internal.h"
 #include "q88.h"
 
+int cm_conv_sc_launch(const int16_t* x, const int16_t* w, const uint8_t* wpk, uint32_t wpk_bytes, uint32_t tb,
+                      uint32_t steps, const int16_t* bias, int16_t* y, uint32_t batch, uint32_t in_ch, uint32_t in_h,
+                      uint32_t in_w, uint32_t out_ch, uint32_t out_h, uint32_t out_w, uint32_t kh, uint32_t kw,
+                      uint32_t sh, uint32_t sw, uint32_t dh, uint32_t dw, uint32_t pt, uint32_t pl,
+                      const EpiArgs& epi, hipStream_t s);
+
 namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
@@ -1243,6 +1249,11 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
     const uint32_t* wsum = reinterpret_cast<const uint32_t*>(wpk + pk_bytes);
     const uint32_t* wfit = wsum + mtiles * TB;
 
+    if (mode == kRunPacked && !pair && in_ch <= 4) {   // the few-channel kernel reads the same planes
+        const int rc = cm_conv_sc_launch(x, nullptr, wpk, (uint32_t)pk_limb, TB, steps, bias, y, batch, in_ch, in_h, in_w,
+                                         out_ch, out_h, out_w, kh, kw, sh, sw, dh, dw, pad_top, pad_left, ea, lc.s);
+        if (rc != 1) return rc;
+    }
     PgArgs g{};
     g.x = x; g.wpk = wpk; g.wsum = wsum; g.wfit = wfit; g.bias = bias; g.y = y;
     g.C = in_ch; g.H = in_h; g.W = in_w; g.M = out_ch; g.OH = out_h; g.OW = out_w; g.P = (uint32_t)P;
