@@ -68,6 +68,20 @@ class TensorLayout:
             return (idx // self.chunk) * self.stride + idx % self.chunk
         return idx
 
+    def view(self, buf):
+        """The tensor's elements of its buffer, in logical order, as a writable view
+        [chunk count, chunk] (`positions` as an index costs an array of 8 bytes per
+        element and a gather through it: 85 us for the 64 x 784 classifier, 43 this way)."""
+        import numpy as np
+        if self.n_chunks <= 1:
+            return buf[:self.numel].reshape(1, self.numel)
+        if self.numel != self.n_chunks * self.chunk:
+            raise ValueError(f"{self.numel} elements are not {self.n_chunks} chunks of {self.chunk}")
+        if len(buf) < (self.n_chunks - 1) * self.stride + self.chunk:
+            raise ValueError(f"{self} does not fit a buffer of {len(buf)}")
+        step = buf.strides[0]
+        return np.lib.stride_tricks.as_strided(buf, (self.n_chunks, self.chunk), (self.stride * step, step))
+
 
 _SPECIAL = (MatmulNode, ConvNode, PoolNode, ReshapeNode)
 
@@ -337,7 +351,8 @@ class BufferPlan:
         for t in self.graph.weight_tensors:
             st = self.storage[t.onnx_name]
             lay = self.layouts[t.onnx_name]
-            img[st.offset + lay.positions()] = t.storage()
+            view = lay.view(img[st.offset:])
+            view[...] = t.storage().reshape(view.shape)
         return img
 
     def scatter(self, name: str, raw, buf) -> None:
@@ -347,14 +362,15 @@ class BufferPlan:
         raw = np.asarray(raw, dtype=np.int16).reshape(-1)
         if raw.size != lay.numel:
             raise ValueError(f"'{name}' needs {lay.numel} values, got {raw.size}")
-        buf[lay.positions()] = raw
+        view = lay.view(buf)
+        view[...] = raw.reshape(view.shape)
 
     def gather(self, name: str, buf):
         """A tensor's logical raw int16 values, in its shape, read from its buffer."""
         import numpy as np
         lay = self.layouts[name]
         shape = self.graph.get_tensor(name).shape
-        return np.asarray(buf)[lay.positions()].astype(np.int16).reshape(shape or [1])
+        return lay.view(np.asarray(buf)).astype(np.int16).reshape(shape or [1])
 
     def summary(self) -> str:
         lines = [f"pool: {self.pool_elems} elements ({self.pool_elems * BYTES_PER_ELEM} B)"]
