@@ -75,12 +75,13 @@ struct PgArgs {
     uint32_t zslot;              // byte offset in each plane of 16 bytes holding the limbs of 0
     uint32_t spos_off, epi_off;  // LDS byte offsets of the position sums and the epilogue tiles
     uint32_t lhc, wr, nh;        // padding columns: left [0, lhc), right [wr, wr + nh - lhc)
+    uint32_t nrun;               // run staging: most 8-element groups of a block's input rows
     uint32_t stage_g;            // 16-byte staging: (row, column group) pair groups per block
     uint32_t cpt_last;           // 16-channel groups of the last chunk
     uint32_t cpt_all;            // without MULTI: 16-channel groups the patch holds (every chunk)
     uint32_t nfull;              // without MULTI: full 64-channel chunks before the last one
     uint32_t L, rpi, rpi_n;      // output pixels per block; ranges per image; ranges per row tile
-    FastDiv div_npr, div_nbm, div_rpi, div_ow, div_npos, div_pw, div_nv, div_prows, div_nh, div_kw, div_cpt4, div_cpt_last, div_t4;
+    FastDiv div_npr, div_nbm, div_rpi, div_ow, div_npos, div_pw, div_nv, div_prows, div_nh, div_kw, div_cpt4, div_cpt_last, div_t4, div_nrun, div_w;
     uint32_t vw;                 // output / Add access width in elements (8 or 1)
     uint32_t add_w4;             // Add runs 4-byte aligned (P even, operand 4-byte aligned)
     uint32_t x_img_bytes, pk_bytes;   // pk_bytes: both packed layouts (limb planes, then int8)
@@ -220,7 +221,11 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// VEC: patch rows loaded 16 bytes at a time with g = VEC; 0 = per element.
+// VEC: how the patch is staged.  1 and 2: rows of whole 16-byte groups, loaded
+// 16 bytes at a time, g = VEC.  3 and 4 (g = 1, any other row): a channel's input
+// rows as one run of 8-element groups counted from the channel's first element;
+// 3 where every channel starts on a dword, 4 where one may not (five dwords,
+// shifted).  0: per element (g = 2 with other rows, g above 2).
 // MULTI: 64-channel chunks restaged in turn inside the k loop (more channels
 // than one patch holds), with fewer loads in flight while the accumulators are
 // live.
@@ -243,6 +248,7 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
     constexpr uint32_t PT = 2u * TB * 64u;        // limb-plane bytes per (row tile, k step)
     constexpr uint32_t PT8 = TB * 64u;            // int8-plane bytes per (row tile, k step)
     constexpr int kPB = MULTI ? 1 : 4;   // 16-byte staging tasks per thread in flight
+    constexpr int kPR = 2;               // run tasks per thread in flight
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ int32_t qtab[kMaxQ + 4];  // per sub-chunk q: patch byte offset of its tap and group
     __shared__ uint32_t tpos[kMaxTaps];  // per tap: patch position offset from a window origin
@@ -286,6 +292,12 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
     const __amdgpu_buffer_rsrc_t wrs = make_rsrc(reinterpret_cast<const int16_t*>(g.wpk), g.pk_bytes);
     const __amdgpu_buffer_rsrc_t wrs2 = make_rsrc(reinterpret_cast<const int16_t*>(g.wpk2), g.pk2_bytes);
     const uint32_t hw_in = g.H * g.W;
+    // run staging: the image from the dword its first element is in, to the end of
+    // the dword its last one is in
+    const uintptr_t ximg = (uintptr_t)(g.x + (uint64_t)n * g.x_img);
+    const uint32_t xodd = VEC == 4 ? (uint32_t)ximg & 2u : 0u;
+    const __amdgpu_buffer_rsrc_t rrs = make_rsrc(reinterpret_cast<const int16_t*>(ximg - xodd),
+                                                 (g.x_img_bytes + xodd + 3u) & ~3u);
 
     if (tid == 0) {   // the zero slot: 16 bytes of each plane holding the limbs of 0
         *reinterpret_cast<v4u*>(p_hi + g.zslot) = v4u{0u, 0u, 0u, 0u};
@@ -388,6 +400,107 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
                     }
                     *reinterpret_cast<uint32_t*>(p_hi + dst[u]) = wh;
                     *reinterpret_cast<uint32_t*>(p_lo + dst[u]) = wl;
+                }
+            }
+        } else if constexpr (VEC >= 3) {
+            // Runs: task e = (channel quad cq, 8-element group v of the input rows the
+            // range touches), four loads (one per channel).  A load is 16 bytes where
+            // the element form's is 2, and a group's elements are placed one by one,
+            // so rows of any length stage alike: 256 -> 256 3x3 at 32 x 14 x 14
+            // 26.0 -> 22.4 us, the MobileNetV2-like graph at batch 16 317 -> 306.  ql
+            // channel quads sit on neighbouring lanes: their LDS writes are neighbouring dwords,
+            // where groups eight positions apart are a multiple of 128 bytes apart
+            // and meet in one or two banks.  Groups count from the channel's first
+            // element, so all four channels' loads start on a dword (VEC 4: on the one
+            // before, by the channel's parity); what a group holds outside the rows
+            // [i_lo, i_hi) of the input is not written, and past the image it reads 0.
+            const int32_t ih_end = ih_first + (int32_t)prows_b;
+            const uint32_t r_lo = ih_first < 0 ? 0u : min((uint32_t)ih_first, g.H);
+            const uint32_t r_hi = ih_end < 0 ? 0u : min((uint32_t)ih_end, g.H);
+            const uint32_t i_lo = r_lo * g.W, i_n = r_hi > r_lo ? (r_hi - r_lo) * g.W : 0u;
+            const uint32_t v_lo = i_lo >> 3, ngrp = i_n ? ((i_lo + i_n + 7u) >> 3) - v_lo : 0u;
+            const uint32_t lql = (uint32_t)__builtin_ctz(ncq | 16u), ql = 1u << lql;
+            const uint32_t ntask = ncq * g.nrun;
+            const uint32_t plane2 = hw_in * 2u;
+            const uint32_t cols = g.PW > g.pl ? g.PW - g.pl : 0u;   // input columns the patch holds
+            const uint32_t wrap = (g.PW - g.W) * g.ppitch;          // (modulo 2^32) from a row's end to the next
+            for (uint32_t b0 = 0; b0 < ntask; b0 += kPgThreads * kPR) {
+                v4u d[kPR][4];
+                uint32_t x5[kPR][4];
+                uint32_t grp[kPR], cql[kPR];
+#pragma unroll
+                for (int u = 0; u < kPR; ++u) {
+                    const uint32_t e = b0 + u * kPgThreads + tid;
+                    const uint32_t rest = e >> lql;
+                    const uint32_t qb = fdiv(rest, g.div_nrun), v = rest - qb * g.nrun;
+                    cql[u] = qb * ql + (e & (ql - 1u));
+                    grp[u] = v_lo + v;
+                    const uint32_t ok = (uint32_t)(e < ntask) & (uint32_t)(v < ngrp);
+                    if (!ok) cql[u] = ncq;
+                    const uint32_t c = c0 + cql[u] * 4u;
+                    const uint32_t base = (c * hw_in + grp[u] * 8u) * 2u + xodd;
+#pragma unroll
+                    for (int jj = 0; jj < 4; ++jj) {
+                        const uint32_t okc = ok & (uint32_t)(c + jj < g.C);
+                        const uint32_t off = ((base + jj * plane2) & 0x7FFFFFFCu) | ((okc ^ 1u) << 31);
+                        d[u][jj] = __builtin_amdgcn_raw_buffer_load_b128(rrs, off, 0, 0);
+                        if constexpr (VEC == 4) x5[u][jj] = __builtin_amdgcn_raw_buffer_load_b32(rrs, off + 16u, 0, 0);
+                    }
+                }
+                // while the first loads are in flight: the positions outside the image
+                if (b0 == 0) {
+                    const uint32_t np = prows_b * g.PW;
+                    for (uint32_t pos = tid; pos < np; pos += kPgThreads) {
+                        const uint32_t r = fdiv(pos, g.div_pw), col = pos - r * g.PW;
+                        if ((uint32_t)(ih_first + (int32_t)r) < g.H && col - g.pl < g.W) continue;
+                        for (uint32_t q = 0; q < cpt; ++q) {
+                            *reinterpret_cast<v4u*>(p_hi + pos * g.ppitch + q * 16u) = v4u{0u, 0u, 0u, 0u};
+                            *reinterpret_cast<v4u*>(p_lo + pos * g.ppitch + q * 16u) =
+                                v4u{0x80808080u, 0x80808080u, 0x80808080u, 0x80808080u};
+                        }
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < kPR; ++u) {
+                    if (cql[u] >= ncq) continue;
+                    const uint32_t el = grp[u] * 8u;
+                    if constexpr (VEC == 4) {
+                        const uint32_t base = ((c0 + cql[u] * 4u) * hw_in + el) * 2u + xodd;
+#pragma unroll
+                        for (int jj = 0; jj < 4; ++jj) {
+                            const uint32_t sh = ((base + jj * plane2) & 2u) * 8u;
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                d[u][jj][k] = __builtin_amdgcn_alignbit(k < 3 ? d[u][jj][k + 1] : x5[u][jj],
+                                                                        d[u][jj][k], sh);
+                        }
+                    }
+                    const uint32_t row = fdiv(el, g.div_w);
+                    uint32_t col = el - row * g.W, i = el - i_lo;   // i: modulo 2^32 below the run
+                    uint32_t dst = (uint32_t)((int32_t)row - ih_first) * g.PW * g.ppitch +
+                                   (col + g.pl) * g.ppitch + cql[u] * 4u;
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const uint32_t d0 = d[u][0][k], d1 = d[u][1][k], d2 = d[u][2][k], d3 = d[u][3][k];
+                        const uint32_t t01 = __builtin_amdgcn_perm(d1, d0, 0x07030501u);
+                        const uint32_t t23 = __builtin_amdgcn_perm(d3, d2, 0x07030501u);
+                        const uint32_t u01 = __builtin_amdgcn_perm(d1, d0, 0x06020400u);
+                        const uint32_t u23 = __builtin_amdgcn_perm(d3, d2, 0x06020400u);
+#pragma unroll
+                        for (int h = 0; h < 2; ++h) {
+                            const uint32_t sel = h ? 0x07060302u : 0x05040100u;
+                            if (i < i_n && col < cols) {
+                                *reinterpret_cast<uint32_t*>(p_hi + dst) = __builtin_amdgcn_perm(t23, t01, sel);
+                                *reinterpret_cast<uint32_t*>(p_lo + dst) =
+                                    __builtin_amdgcn_perm(u23, u01, sel) ^ 0x80808080u;
+                            }
+                            ++i;
+                            ++col;
+                            const bool over = col == g.W;
+                            dst += g.ppitch + (over ? wrap : 0u);
+                            col = over ? 0u : col;
+                        }
+                    }
                 }
             }
         } else {
@@ -1280,6 +1393,10 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
         g.stage_g = npr < kPgThreads ? kPgThreads / npr : 1u;
         g.div_npr = make_fastdiv(npr);
     }
+    // a run of prows * W elements starting anywhere in a group
+    g.nrun = (uint32_t)std::min<uint64_t>(prows * in_w + 14u, (uint64_t)in_h * in_w + 7u) / 8u;
+    g.div_nrun = make_fastdiv(g.nrun);
+    g.div_w = make_fastdiv(in_w);
     g.div_prows = make_fastdiv((uint32_t)prows);
     g.div_nh = make_fastdiv(nh ? nh : 1);
     g.div_kw = make_fastdiv(kw);
@@ -1311,8 +1428,11 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
     g.vw = P % 8 == 0 && aligned(y, 16) && (ea.add_mode != 1u || aligned(ea.add, 16)) ? 8u : 1u;
     g.add_w4 = P % 2 == 0 && ea.add_mode == 1u && aligned(ea.add, 4) ? 1u : 0u;
     const void* k = nullptr;
-#define CM_PG_PICK(M, NS, W, PR) (vec == 1 ? (const void*)conv_pgemm<1, M, NS, W, PR> \
-                                  : vec == 2 ? (const void*)conv_pgemm<2, M, NS, W, PR> \
+    const uint32_t st = vec || gg != 1u ? vec : (uint64_t)in_h * in_w % 2 == 0 && aligned(x, 4) ? 3u : 4u;
+#define CM_PG_PICK(M, NS, W, PR) (st == 1 ? (const void*)conv_pgemm<1, M, NS, W, PR> \
+                                  : st == 2 ? (const void*)conv_pgemm<2, M, NS, W, PR> \
+                                  : st == 3 ? (const void*)conv_pgemm<3, M, NS, W, PR> \
+                                  : st == 4 ? (const void*)conv_pgemm<4, M, NS, W, PR> \
                                              : (const void*)conv_pgemm<0, M, NS, W, PR>)
 #define CM_PG_PICK_W(M, NS, PR) (wrows == 1 ? CM_PG_PICK(M, NS, 1, PR) : wrows == 2 ? CM_PG_PICK(M, NS, 2, PR) \
                                                                              : CM_PG_PICK(M, NS, 4, PR))
