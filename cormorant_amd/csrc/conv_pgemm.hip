@@ -54,6 +54,7 @@ namespace {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned int v4u __attribute__((ext_vector_type(4)));
+typedef v4u v4u_a4 __attribute__((aligned(4)));   // 16-byte accesses from any dword
 
 constexpr uint32_t kMaxTB = 128;   // output channels per row tile: 32, 64 or 128
 constexpr int kMaxQ = 256;                    // q table entries (taps * 4 <= 256)
@@ -82,8 +83,8 @@ struct PgArgs {
     uint32_t nfull;              // without MULTI: full 64-channel chunks before the last one
     uint32_t L, rpi, rpi_n;      // output pixels per block; ranges per image; ranges per row tile
     FastDiv div_npr, div_nbm, div_rpi, div_ow, div_npos, div_pw, div_nv, div_prows, div_nh, div_kw, div_cpt4, div_cpt_last, div_t4, div_nrun, div_w;
-    uint32_t vw;                 // output / Add access width in elements (8 or 1)
-    uint32_t add_w4;             // Add runs 4-byte aligned (P even, operand 4-byte aligned)
+    uint32_t y_w4;               // output runs start on a dword (P even, y 4-byte aligned)
+    uint32_t add_w4;             // Add runs start on a dword (P even, operand 4-byte aligned)
     uint32_t x_img_bytes, pk_bytes;   // pk_bytes: both packed layouts (limb planes, then int8)
     uint32_t pk8_off;            // byte offset of the int8 plane
     uint64_t x_img, y_img;
@@ -635,10 +636,9 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
     // m_end on read 0; pixels p0w.. of the range, pnw of them valid), laid out as
     // finish_tile reads them (half i, run t: row (lane / 8) + 8t of the half,
     // pixels 8 * (lane % 8)..+8, as 8 packed int16), loaded ahead of the finish
-    // in one go: 16-byte loads when the runs are 16-byte aligned, 4-byte loads
-    // when they are 4-byte aligned, else 2-byte loads.  Values past a run's valid
-    // pixels are never stored (they lie in the operand's image, or past it,
-    // where the buffer reads 0); empty runs and rows past m_end read 0 through
+    // in one go: 16-byte loads when the runs start on a dword, else 2-byte loads.
+    // Values past a run's valid pixels are never stored (they lie in the operand's
+    // image, or past it, where the buffer reads 0 dword by dword); empty runs and rows past m_end read 0 through
     // bit 31 of their offset, never through a branch.  Every load is issued
     // before any is used.
     const __amdgpu_buffer_rsrc_t ars = make_rsrc(g.epi.add_mode == 1u ? g.epi.add + (uint64_t)n * g.y_img : g.x,
@@ -654,19 +654,11 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
                 const uint32_t bad = (uint32_t)(m >= m_end || c8 >= pnw);
                 off[i][t] = ((m * g.P + p0w + c8) * 2u) | (bad << 31);
             }
-        if (g.vw == 8u) {
+        if (g.add_w4) {
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int t = 0; t < 2; ++t) av[i][t] = __builtin_amdgcn_raw_buffer_load_b128(ars, off[i][t], 0, 0);
-        } else if (g.add_w4) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int t = 0; t < 2; ++t)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q)
-                        av[i][t][q] = __builtin_amdgcn_raw_buffer_load_b32(ars, off[i][t] + 4u * q, 0, 0);
         } else {
             uint32_t h[2][2][8];
 #pragma unroll
@@ -716,9 +708,9 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
                     const uint64_t o = (uint64_t)n * g.y_img + (uint64_t)m * g.P + p0w + c8;
                     const v4u tv = *reinterpret_cast<const v4u*>(et + r * kEpiPitch + c8);
                     int16_t* yp = g.y + o;
-                    const bool vec8 = ncol == 8u && g.vw == 8u;
+                    const bool vec8 = ncol == 8u && g.y_w4;
                     if (plain && vec8) {
-                        *reinterpret_cast<v4u*>(yp) = tv;
+                        *reinterpret_cast<v4u_a4*>(yp) = tv;
                         continue;
                     }
                     int32_t yv[8];
@@ -737,7 +729,7 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
 #pragma unroll
                     for (int q = 0; q < 8; ++q) yv[q] = q88::clamp(yv[q], lo, hi);
                     if (vec8) {
-                        *reinterpret_cast<v4u*>(yp) = v4u{pack2(yv[0], yv[1]), pack2(yv[2], yv[3]),
+                        *reinterpret_cast<v4u_a4*>(yp) = v4u{pack2(yv[0], yv[1]), pack2(yv[2], yv[3]),
                                                           pack2(yv[4], yv[5]), pack2(yv[6], yv[7])};
                     } else {
 #pragma unroll
@@ -1423,9 +1415,12 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
         g.pk2_8off = (uint32_t)pk2_limb;
         g.act1 = pair->act1;
     }
-    // 16-byte output accesses: every run of 8 pixels starts 16-byte aligned
-    // (ranges start at multiples of L, sub-tiles at multiples of 64 pixels)
-    g.vw = P % 8 == 0 && aligned(y, 16) && (ea.add_mode != 1u || aligned(ea.add, 16)) ? 8u : 1u;
+    // 16-byte output and Add accesses wherever a run of 8 pixels starts on a dword
+    // (ranges start at multiples of L, sub-tiles at multiples of 64 pixels): planes
+    // that are even but not whole groups stored element by element before, 256 -> 256 3x3
+    // at 32 x 14 x 14 22.4 -> 21.3 us, 24 -> 344 7x7 at 20 x 18 x 18 35.7 -> 33.1.
+    // At odd elements wide accesses are the slower ones.
+    g.y_w4 = P % 2 == 0 && aligned(y, 4) ? 1u : 0u;
     g.add_w4 = P % 2 == 0 && ea.add_mode == 1u && aligned(ea.add, 4) ? 1u : 0u;
     const void* k = nullptr;
     const uint32_t st = vec || gg != 1u ? vec : (uint64_t)in_h * in_w % 2 == 0 && aligned(x, 4) ? 3u : 4u;
