@@ -249,7 +249,9 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
     constexpr uint32_t PT = 2u * TB * 64u;        // limb-plane bytes per (row tile, k step)
     constexpr uint32_t PT8 = TB * 64u;            // int8-plane bytes per (row tile, k step)
     constexpr int kPB = MULTI ? 1 : 4;   // 16-byte staging tasks per thread in flight
-    constexpr int kPR = 2;               // run tasks per thread in flight
+    // run tasks per thread in flight (beside live accumulators two spilled 66 registers:
+    // 512 -> 512 3x3 at 32 x 7 x 7 132 us, 34.5 with one)
+    constexpr int kPR = MULTI ? 1 : 2;
     extern __shared__ __align__(16) uint8_t lds[];
     __shared__ int32_t qtab[kMaxQ + 4];  // per sub-chunk q: patch byte offset of its tap and group
     __shared__ uint32_t tpos[kMaxTaps];  // per tap: patch position offset from a window origin
@@ -1423,7 +1425,11 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
     g.y_w4 = P % 2 == 0 && aligned(y, 4) ? 1u : 0u;
     g.add_w4 = P % 2 == 0 && ea.add_mode == 1u && aligned(ea.add, 4) ? 1u : 0u;
     const void* k = nullptr;
-    const uint32_t st = vec || gg != 1u ? vec : (uint64_t)in_h * in_w % 2 == 0 && aligned(x, 4) ? 3u : 4u;
+    // Rows of other lengths as runs; restaged chunks of planes below 128 elements whose
+    // channels start between dwords stay on element loads: 512 -> 512 3x3 at 32 x 7 x 7
+    // 33.6 us against 34.5, at 8 x 15 x 15 41.8 against 35.5.
+    const uint64_t hw = (uint64_t)in_h * in_w;
+    const uint32_t st = vec || gg != 1u ? vec : hw % 2 == 0 && aligned(x, 4) ? 3u : multi && hw < 128 ? 0u : 4u;
 #define CM_PG_PICK(M, NS, W, PR) (st == 1 ? (const void*)conv_pgemm<1, M, NS, W, PR> \
                                   : st == 2 ? (const void*)conv_pgemm<2, M, NS, W, PR> \
                                   : st == 3 ? (const void*)conv_pgemm<3, M, NS, W, PR> \
