@@ -87,6 +87,7 @@ struct PgArgs {
     uint32_t add_w4;             // Add runs start on a dword (P even, operand 4-byte aligned)
     uint32_t x_img_bytes, pk_bytes;   // pk_bytes: both packed layouts (limb planes, then int8)
     uint32_t pk8_off;            // byte offset of the int8 plane
+    uint32_t pk_rows;            // rows of a packed row tile (TB, or more when the layer has one tile)
     uint64_t x_img, y_img;
     EpiArgs epi;
     // PAIR: a 1x1 convolution (M2 output channels) applied to this convolution's
@@ -246,8 +247,8 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
     constexpr uint32_t TB = 32u * WR;             // output channels per row tile
     constexpr uint32_t WC = 4u / WR;              // wave columns
     constexpr uint32_t SPX = 64u * WC;            // pixels per sub-tile
-    constexpr uint32_t PT = 2u * TB * 64u;        // limb-plane bytes per (row tile, k step)
-    constexpr uint32_t PT8 = TB * 64u;            // int8-plane bytes per (row tile, k step)
+    const uint32_t PT8 = g.pk_rows * 64u;         // int8-plane bytes per (row tile, k step)
+    const uint32_t PT = 2u * PT8;                 // limb-plane bytes per (row tile, k step)
     constexpr int kPB = MULTI ? 1 : 4;   // 16-byte staging tasks per thread in flight
     // run tasks per thread in flight (beside live accumulators two spilled 66 registers:
     // 512 -> 512 3x3 at 32 x 7 x 7 132 us, 34.5 with one)
@@ -317,7 +318,7 @@ __global__ __launch_bounds__(kPgThreads, 2) void conv_pgemm(PgArgs g) {
         for (int i = 0; i < 2; ++i) {
             ah[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(wrs, off + i * 1024u, 0, 0));
             al[i] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(
-                wrs, off + TB * 64u + i * 1024u, 0, 0));
+                wrs, off + PT8 + i * 1024u, 0, 0));
         }
     };
     // the int8 plane's A fragments of step gs (rows whose weights all fit int8)
@@ -1184,8 +1185,16 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
         in_w >= (1u << 20) || out_w > 4096 || pad_top >= in_h + kh * dh || pad_left >= in_w + kw * dw)
         return 1;
     const uint32_t nchunks = (in_ch + 63) / 64;
-    // row tile: 32, 64 or 128 output channels (128 with several channel chunks)
-    const uint32_t wrows = nchunks > 1 || out_ch > 64 ? 4u : out_ch > 32 ? 2u : 1u;
+    // row tile: 32, 64 or 128 output channels, the smallest that holds them all.  The
+    // weights of several channel chunks are packed in 128-row tiles whatever the layer
+    // has; it runs on a smaller tile when its wave columns (128 or 256 pixels a
+    // sub-tile) find 64 sub-tiles: 128 -> 32 3x3 at 32 x 56 x 56 41.3 -> 26.2 us,
+    // 28 x 28 14.8 -> 13.3, 100 -> 60 5x5 at 16 x 40 x 40 25.5 -> 22.0, but 256 -> 64
+    // 3x3 at 16 x 14 x 14 (25 sub-tiles) 12.0 -> 12.5.
+    const uint32_t least = out_ch > 64 ? 4u : out_ch > 32 ? 2u : 1u;
+    const uint32_t pack_rows = 32u * (nchunks > 1 ? 4u : least);
+    const bool narrow = !pair && (uint64_t)batch * P >= 64ull * (256u / least);
+    const uint32_t wrows = nchunks > 1 && !narrow ? 4u : least;
     const uint32_t TB = 32u * wrows, SPX = 256u / wrows;
     const uint32_t mtiles = (out_ch + TB - 1) / TB;
     const uint32_t gg = gcd(sh, dh), Sg = sh / gg, Dg = dh / gg;
@@ -1245,7 +1254,7 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
         const uint64_t c_row = (uint64_t)PW * cpt_row * 2;
         uint32_t l_best = 0;
         uint64_t best = ~0ull;
-        const uint64_t lcap = multi ? 128u : 512u;
+        const uint64_t lcap = multi ? 2u * SPX : 512u;
         for (uint64_t l = 16; l <= lcap; l += 16) {
             // output rows a range spans: ranges start at multiples of l, so a
             // range's offset within its first row is a multiple of gcd(l, out_w),
@@ -1311,15 +1320,16 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
     const uint64_t zslot = prows * PW * ppitch;
     const uint64_t p_plane = zslot + 16;
     // workspace: limb planes, int8 plane, row sums, int8 flags
-    const uint64_t pk_limb = (uint64_t)mtiles * steps * (2u * TB * 64u);
-    const uint64_t pk_bytes = pk_limb + (uint64_t)mtiles * steps * (TB * 64u);
+    const uint32_t prow_n = (out_ch + pack_rows - 1) / pack_rows * pack_rows;   // packed rows
+    const uint64_t pk_limb = (uint64_t)prow_n * steps * 128u;
+    const uint64_t pk_bytes = pk_limb + (uint64_t)prow_n * steps * 64u;
     // pair: the 1x1's packed weights after the first convolution's (32-row
     // tiles, the same plane layout with one tap), then its row sums and flags
     const uint32_t mtiles2 = (m2 + 31u) / 32u;
-    const uint64_t off2 = pair ? (pk_bytes + 8ull * mtiles * TB + 255u) & ~255ull : 0u;
+    const uint64_t off2 = pair ? (pk_bytes + 8ull * prow_n + 255u) & ~255ull : 0u;
     const uint64_t pk2_limb = (uint64_t)mtiles2 * steps2 * (2u * 32u * 64u);
     const uint64_t pk2_bytes = pk2_limb + (uint64_t)mtiles2 * steps2 * (32u * 64u);
-    const uint64_t need = pair ? off2 + pk2_bytes + 8ull * mtiles2 * 32u : pk_bytes + 8ull * mtiles * TB;
+    const uint64_t need = pair ? off2 + pk2_bytes + 8ull * mtiles2 * 32u : pk_bytes + 8ull * prow_n;
     if (pk_bytes >= 0x80000000ull) return 1;
     if (lc.need) {
         if (need > *lc.need) *lc.need = need;
@@ -1338,9 +1348,9 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
             return 1;
         }
         PackArgs pa{w, wbuf, wbuf + pk_limb, reinterpret_cast<uint32_t*>(wbuf + pk_bytes),
-                    reinterpret_cast<uint32_t*>(wbuf + pk_bytes) + mtiles * TB,
-                    in_ch, out_ch, taps, nchunks, steps, taps, TB};
-        hipLaunchKernelGGL(conv_wpack, dim3(mtiles * TB), dim3(256), 0, lc.s, pa);
+                    reinterpret_cast<uint32_t*>(wbuf + pk_bytes) + prow_n,
+                    in_ch, out_ch, taps, nchunks, steps, taps, pack_rows};
+        hipLaunchKernelGGL(conv_wpack, dim3(prow_n), dim3(256), 0, lc.s, pa);
         int rc = cm_check_launch("conv_wpack");
         if (!rc && pair) {
             uint8_t* w2 = wbuf + off2;
@@ -1354,10 +1364,10 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
     }
     const uint8_t* wpk = mode == kRunPacked ? static_cast<const uint8_t*>(packed) : wbuf;
     const uint32_t* wsum = reinterpret_cast<const uint32_t*>(wpk + pk_bytes);
-    const uint32_t* wfit = wsum + mtiles * TB;
+    const uint32_t* wfit = wsum + prow_n;
 
     if (mode == kRunPacked && !pair && in_ch <= 4) {   // the few-channel kernel reads the same planes
-        const int rc = cm_conv_sc_launch(x, nullptr, wpk, (uint32_t)pk_limb, TB, steps, bias, y, batch, in_ch, in_h, in_w,
+        const int rc = cm_conv_sc_launch(x, nullptr, wpk, (uint32_t)pk_limb, pack_rows, steps, bias, y, batch, in_ch, in_h, in_w,
                                          out_ch, out_h, out_w, kh, kw, sh, sw, dh, dw, pad_top, pad_left, ea, lc.s);
         if (rc != 1) return rc;
     }
@@ -1400,6 +1410,7 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
     g.x_img_bytes = (uint32_t)(2 * x_img);
     g.pk_bytes = (uint32_t)pk_bytes;
     g.pk8_off = (uint32_t)pk_limb;
+    g.pk_rows = pack_rows;
     g.x_img = x_img;
     g.y_img = (uint64_t)(pair ? m2 : out_ch) * P;
     g.epi = ea;
@@ -1437,7 +1448,7 @@ int pg_launch(const int16_t* x, const int16_t* w, const int16_t* bias, int16_t* 
                                              : (const void*)conv_pgemm<0, M, NS, W, PR>)
 #define CM_PG_PICK_W(M, NS, PR) (wrows == 1 ? CM_PG_PICK(M, NS, 1, PR) : wrows == 2 ? CM_PG_PICK(M, NS, 2, PR) \
                                                                              : CM_PG_PICK(M, NS, 4, PR))
-    if (multi) k = CM_PG_PICK(true, 2, 4, false);
+    if (multi) k = CM_PG_PICK_W(true, 2, false);
     else if (pair) k = steps % 3 == 0 ? CM_PG_PICK_W(false, 3, true) : CM_PG_PICK_W(false, 2, true);
     else if (steps % 3 == 0) k = CM_PG_PICK_W(false, 3, false);
     else k = CM_PG_PICK_W(false, 2, false);

@@ -23,6 +23,9 @@ CASES = [
     (1, 66, 12, 100, 65, 1, 3, 1, 1, 0, 2, 2), (4, 70, 5, 3, 66, 3, 3, 1, 1, 1, 1, 1),
     (2, 68, 1, 6, 72, 1, 2, 1, 1, 0, 1, 1), (2, 66, 23, 1, 66, 2, 1, 1, 1, 0, 0, 0),
     (1, 80, 18, 21, 70, 3, 3, 1, 2, 2, 2, 2), (2, 67, 6, 6, 65, 3, 3, 1, 1, 5, 4, 3),
+    # several channel chunks on 32- and 64-row tiles, one patch and restaged
+    (21, 70, 28, 28, 31, 3, 3, 1, 1, 1, 1, 1), (11, 130, 28, 27, 33, 3, 3, 1, 1, 1, 1, 1),
+    (84, 600, 14, 14, 20, 3, 3, 1, 1, 1, 1, 1), (3, 81, 56, 56, 64, 3, 3, 1, 1, 1, 1, 1),
     (1, 64, 15, 129, 96, 3, 3, 1, 1, 1, 1, 1), (2, 7, 63, 63, 90, 7, 7, 1, 1, 3, 3, 3),
 ]
 
